@@ -252,7 +252,10 @@ def require_device(t: torch.Tensor, what: str) -> None:
 
 def stream_of(device: torch.device) -> int:
     """Handle of torch's current stream (without the Stream object that
-    torch.cuda.current_stream makes: 0.3 instead of 3 us)."""
+    torch.cuda.current_stream makes: 0.3 instead of 3 us).  Refuses other
+    devices as that does: what is launched next would read host addresses."""
+    if device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
