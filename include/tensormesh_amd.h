@@ -688,9 +688,10 @@ int tm_pcg_iterate(const tm_pcg_view* view, void* x, int32_t n_iter, tm_stream_t
  * Workgroups of a system wait for each other (they are launched
  * cooperatively).  A launch ends without a result, with the int32 at the
  * last 16 bytes of the first tm_pcg_run_bytes of ws nonzero, when a wait
- * takes more than 2 s (1) or a workgroup reads more than 4,096 columns of
- * others (2); solve from the initial guess again, by tm_pcg_iterate.  No
- * counterpart in the reference. */
+ * takes more than 2 s (1), a workgroup reads more than 4,096 columns of
+ * others (2), or a row has more than plan->row_entries entries or a column
+ * outside its system (3); solve from the initial guess again, by
+ * tm_pcg_iterate.  No counterpart in the reference. */
 typedef struct tm_pcg_run_plan {
   int64_t n_wg, n_solo;
   const int32_t* wg_sys;      /* [n_wg] system of the workgroup */

@@ -158,6 +158,7 @@ __global__ void __launch_bounds__(kThreads) cg2_run_kernel(RunArgs a) {
   if (c[6] == 0.0) return;  // stopped at its initial residual; cleared later only after every workgroup took part
   if (tid == 0) s_abort = s_halo = 0;
   const int32_t own = a.blk_row0[wb0];  // the workgroup's rows are consecutive
+  const int32_t sys_row0 = a.blk_row0[b0], sys_rows = a.blk_row1[b1 - 1] - sys_row0;
 
   T av[kReg], x[K], r[K], p[K], s[K], w[K], d[K], u[K];
   int32_t row[K], ra[K], len[K];  // row -1: none
@@ -226,15 +227,20 @@ __global__ void __launch_bounds__(kThreads) cg2_run_kernel(RunArgs a) {
     return;
   }
   // byte offsets into s_u of the columns, two to a word; past the row's end
-  // (and without a row) the workgroup's first row
+  // (and without a row) the workgroup's first row.  A row of more entries than
+  // a thread holds, or a column of another system, ends the launch: the first
+  // would be cut short, the second has no place in s_u.
   uint32_t cj[K][PER / 2];
+  bool unfit = false;
 #pragma unroll
-  for (int k = 0; k < K; ++k)
+  for (int k = 0; k < K; ++k) {
+    unfit |= len[k] > PER;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       uint32_t at = 0;
       if (j < len[k]) {
         const int32_t col = a.ci[ra[k] + j];
+        unfit |= (uint32_t)(col - sys_row0) >= (uint32_t)sys_rows;
         at = (uint32_t)(col - own);
         if (!SOLO && at >= (uint32_t)kOwn) {
           uint32_t h = hash(col);
@@ -245,6 +251,8 @@ __global__ void __launch_bounds__(kThreads) cg2_run_kernel(RunArgs a) {
       at *= (uint32_t)sizeof(T);
       cj[k][j / 2] = j % 2 ? cj[k][j / 2] | (at << 16) : at;
     }
+  }
+  if (unfit) s_abort = 1;
   // this thread's halo columns, as byte offsets into a buffer of u
   constexpr int kHaloPer = SOLO ? 1 : kHalo / kThreads;
   uint32_t hc[kHaloPer];
@@ -265,6 +273,10 @@ __global__ void __launch_bounds__(kThreads) cg2_run_kernel(RunArgs a) {
   bool active = true;
   int buf = 0;
   __syncthreads();  // s_red and the tables are read
+  if (s_abort) {    // uniform per workgroup
+    if (tid == 0) post(a.abort, 3);
+    return;
+  }
 #pragma unroll
   for (int k = 0; k < K; ++k)
 #pragma unroll

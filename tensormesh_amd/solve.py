@@ -228,7 +228,7 @@ class BatchedPCG:
         nat.check(nat.lib().tm_pcg_run(ctypes.byref(view), ctypes.byref(plan), self.x.data_ptr(), n,
                                        nat.stream_of(self.dev)), "tm_pcg_run")
         tail = plan._keep[1][plan.ws_bytes - 16:].cpu()
-        if plan.n_launch > 0 and int(tail[:4].view(torch.int32)) != 0:
+        if int(tail[:4].view(torch.int32)) != 0:
             return None
         return tail[16:].view(torch.float64).view(self.n_sys, self.stride)
 

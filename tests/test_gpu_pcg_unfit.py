@@ -1,0 +1,62 @@
+"""Systems that a whole-solve launch (tm_pcg_run) cannot hold end it without a
+result, and the two-launch steps solve them: the same bits as with ``chunk``,
+which asks for those steps."""
+import numpy as np
+import pytest
+import torch
+
+import tensormesh_amd as tm
+from tensormesh_amd.mesh import unit_cube_tet, unit_square_tri
+from tensormesh_amd.solve import BatchedPCG
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _laplace(mesh):
+    m = mesh.to(DEV)
+    K = tm.LaplaceElementAssembler.from_mesh(m)()
+    return tm.Condenser(m.boundary_mask)(K, torch.ones(m.n_points, dtype=torch.float64, device=DEV))
+
+
+def _falls_back(s, f, want):
+    assert s._run_plan() is not None
+    for x, y in zip(s.solve(f), want):
+        assert torch.equal(x, y)
+    assert s._run is None   # found out by that solve
+
+
+# 8 entries per thread, rows of up to 15: one workgroup, and several
+@pytest.mark.parametrize("n", [8, 17])
+def test_rows_longer_than_the_plan(n):
+    print(f"case long rows {n}", flush=True)
+    K, f = _laplace(unit_cube_tet(n, 0.15, 1))
+    assert int((K.row_ptr[1:] - K.row_ptr[:-1]).max()) > 8
+    a, b = (BatchedPCG(K.row_ptr, K.col_indices, K.values, [0, K.shape[0]], rtol=1e-10) for _ in range(2))
+    want = a.solve(f, chunk=32)
+    wgs = -(-np.diff(b._sys_blk) // 4)
+    b._run = b._make_plan(1, 8, int(wgs.max()), wgs)
+    assert (b._run.n_launch == 0) == (K.shape[0] <= 1024)
+    _falls_back(b, f, want)
+
+
+# two systems of 361 rows (a workgroup each), and of 6,241 (several), of which
+# the first has an entry in a column of the second and the other way round
+@pytest.mark.parametrize("n", [20, 80])
+def test_columns_of_another_system(n):
+    print(f"case columns of another system {n}", flush=True)
+    K, f = _laplace(unit_square_tri(n, 0.2, 1))
+    N = K.shape[0]
+    assert N == (n - 1) ** 2
+    last = torch.tensor([N - 1], device=DEV)
+    row = torch.cat([K.row_indices, K.row_indices + N, last, last + 1])
+    col = torch.cat([K.col_indices, K.col_indices + N, last + 1, last])
+    val = torch.cat([K.values, K.values, torch.full((2,), -1e-3, dtype=torch.float64, device=DEV)])
+    order = torch.argsort(row * 2 * N + col)
+    rp = torch.zeros(2 * N + 1, dtype=torch.int64, device=DEV)
+    rp[1:] = torch.cumsum(torch.bincount(row, minlength=2 * N), 0)
+    a, b = (BatchedPCG(rp, col[order], val[order], [0, N, 2 * N], rtol=1e-10) for _ in range(2))
+    ff = torch.cat([f, 2 * f])
+    want = a.solve(ff, chunk=32)
+    assert torch.isfinite(want[0]).all()
+    _falls_back(b, ff, want)
