@@ -206,6 +206,9 @@ SIGNATURES = {
 _LIB: Optional[ctypes.CDLL] = None
 
 
+TM_ERR_HIP, TM_ERR_UNSUPPORTED = -3, -4
+
+
 class NativeError(RuntimeError):
     pass
 

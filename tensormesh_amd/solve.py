@@ -236,8 +236,11 @@ class BatchedPCG:
         None if it ended without a result.  The status word and the scalars are
         neighbours in memory: those of few systems come over in one copy."""
         view, plan = self._view(), self._run
-        nat.check(nat.lib().tm_pcg_run(ctypes.byref(view), ctypes.byref(plan), self.x.data_ptr(), n,
-                                       nat.stream_of(self.dev)), "tm_pcg_run")
+        status = nat.lib().tm_pcg_run(ctypes.byref(view), ctypes.byref(plan), self.x.data_ptr(), n,
+                                      nat.stream_of(self.dev))
+        if status in (nat.TM_ERR_HIP, nat.TM_ERR_UNSUPPORTED):
+            return None   # this device, now, does not take the cooperative launch
+        nat.check(status, "tm_pcg_run")
         whole = self.n_sys <= self.HOST_SYSTEMS
         tail = plan._keep[1][plan.ws_bytes - 16:None if whole else plan.ws_bytes].cpu()
         if int(tail[:4].view(torch.int32)) != 0:

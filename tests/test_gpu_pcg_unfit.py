@@ -6,6 +6,7 @@ import pytest
 import torch
 
 import tensormesh_amd as tm
+from tensormesh_amd import _native as nat
 from tensormesh_amd.mesh import unit_cube_tet, unit_square_tri
 from tensormesh_amd.solve import BatchedPCG
 
@@ -60,3 +61,29 @@ def test_columns_of_another_system(n):
     want = a.solve(ff, chunk=32)
     assert torch.isfinite(want[0]).all()
     _falls_back(b, ff, want)
+
+
+class _Lib:
+    """The library, with ``tm_pcg_run`` ending in a status of its own."""
+
+    def __init__(self, lib, status):
+        self._lib, self._status, self.calls = lib, status, 0
+
+    def __getattr__(self, name):
+        return getattr(self._lib, name)
+
+    def tm_pcg_run(self, *args):
+        self.calls += 1
+        return self._status
+
+
+@pytest.mark.parametrize("name", ["TM_ERR_HIP", "TM_ERR_UNSUPPORTED"])
+def test_a_refused_launch(name, monkeypatch):
+    print(f"case refused launch {name}", flush=True)
+    K, f = _laplace(unit_square_tri(60, 0.2, 1))
+    a, b = (BatchedPCG(K.row_ptr, K.col_indices, K.values, [0, K.shape[0]], rtol=1e-10) for _ in range(2))
+    want = a.solve(f, chunk=32)
+    lib = _Lib(nat.lib(), getattr(nat, name))
+    monkeypatch.setattr(nat, "lib", lambda: lib)
+    _falls_back(b, f, want)
+    assert lib.calls == 1
