@@ -172,6 +172,11 @@ class BatchedPCG:
     #: (rows per thread, entries per row) tm_pcg_run is built for
     RUN_SHAPES = ((1, 8), (1, 16), (1, 24), (2, 8))
 
+    #: Most steps of one launch (1 to 4 s): a kernel can be neither looked at nor
+    #: interrupted, and its step count is 32 bits.  A larger budget that is not
+    #: used up costs nothing; one that is starts over in chunks.
+    RUN_MAX_STEPS = 1 << 18
+
     def _run_plan(self) -> Optional[nat.PcgRunPlan]:
         """Workgroups of ``tm_pcg_run`` (whole solves, a group of systems per
         launch), or None where the stack does not fit it: a row of more
@@ -289,11 +294,14 @@ class BatchedPCG:
         g = sc = None
         if plan is not None:
             steps = -(-max_iter // chunk) * chunk
-            sc = self._run_steps(steps)
+            sc = self._run_steps(min(steps, self.RUN_MAX_STEPS))
+            if sc is None:
+                self._run = None
+            elif steps > self.RUN_MAX_STEPS and bool((sc[:, 6] != 0).any()):
+                sc = None
             if sc is not None:
                 done = steps
             else:
-                self._run = None
                 if x0 is None:
                     self.x.zero_()
                 else:

@@ -87,3 +87,24 @@ def test_a_refused_launch(name, monkeypatch):
     monkeypatch.setattr(nat, "lib", lambda: lib)
     _falls_back(b, f, want)
     assert lib.calls == 1
+
+
+@pytest.mark.parametrize("n", [20, 60])   # one workgroup, and several
+def test_budgets_beyond_one_launch(n, monkeypatch):
+    """A budget past 32 bits is no limit to a solve that converges; one past the
+    steps of a launch goes on in chunks."""
+    print(f"case budgets {n}", flush=True)
+    K, f = _laplace(unit_square_tri(n, 0.2, 1))
+    a, b = (BatchedPCG(K.row_ptr, K.col_indices, K.values, [0, K.shape[0]], rtol=1e-10) for _ in range(2))
+    want = a.solve(f, chunk=32)
+    for max_iter in (2 ** 31, 2 ** 32 + 64, 10 ** 12):
+        for x, y in zip(b.solve(f, max_iter=max_iter), want):
+            assert torch.equal(x, y)
+    assert b._run is not None and int(want[1]) > 32
+    monkeypatch.setattr(BatchedPCG, "RUN_MAX_STEPS", 32)
+    x0 = torch.linspace(-1, 1, K.shape[0], dtype=torch.float64, device=DEV)
+    for kw in ({}, {"max_iter": 32}, {"max_iter": 64}, {"x0": x0}):
+        want = a.solve(f, chunk=32, **kw)
+        for x, y in zip(b.solve(f, **kw), want):
+            assert torch.equal(x, y)
+    assert b._run is not None
