@@ -180,8 +180,9 @@ class BatchedPCG:
     def _run_plan(self) -> Optional[nat.PcgRunPlan]:
         """Workgroups of ``tm_pcg_run`` (whole solves, a group of systems per
         launch), or None where the stack does not fit it: a row of more
-        entries than a thread holds, or a system of more workgroups than run
-        at once."""
+        entries than a thread holds, a system of more workgroups than run at
+        once, or no memory left for the words they exchange (a solve without
+        them takes none beyond the solver's vectors)."""
         if self._run is False:
             self._run = None
             if self.variant == 1 and self.n:
@@ -200,7 +201,10 @@ class BatchedPCG:
                     # thread, 16.4 with one), then few rows per thread (a
                     # 261,121-row system: 5.0 us per step with one, 5.3 with two)
                     _, _, k, per, wgs, most = min(shapes, key=lambda s: s[:4])
-                    self._run = self._make_plan(k, per, most, wgs)
+                    try:
+                        self._run = self._make_plan(k, per, most, wgs)
+                    except torch.OutOfMemoryError:
+                        pass
         return self._run
 
     def _make_plan(self, k: int, per: int, most: int, wgs: np.ndarray) -> nat.PcgRunPlan:

@@ -108,3 +108,20 @@ def test_budgets_beyond_one_launch(n, monkeypatch):
         for x, y in zip(b.solve(f, **kw), want):
             assert torch.equal(x, y)
     assert b._run is not None
+
+
+def test_no_memory_for_the_workspace(monkeypatch):
+    print("case no memory for the workspace", flush=True)
+    K, f = _laplace(unit_square_tri(60, 0.2, 1))
+    a, b = (BatchedPCG(K.row_ptr, K.col_indices, K.values, [0, K.shape[0]], rtol=1e-10) for _ in range(2))
+    want = a.solve(f, chunk=32)
+    empty = torch.empty
+
+    def full(*args, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError("no memory")
+        return empty(*args, **kw)
+    monkeypatch.setattr(torch, "empty", full)
+    for x, y in zip(b.solve(f), want):
+        assert torch.equal(x, y)
+    assert b._run is None
