@@ -42,14 +42,32 @@ __device__ __forceinline__ int64_t xcd_chunks(int64_t b, int64_t nb) {
   return (g + 1) * 8 * kChunk > nb ? b : g * 8 * kChunk + (r % 8) * kChunk + r / 8;
 }
 
+// Nodes per side of the tile of node pairs that a lane owns, for B nodes on L
+// lanes and rules of at most MQ points.  A 2 x 2 tile reads four gradients for
+// four pairs where single pairs read eight, so it is the better one where
+// there are tiles for most lanes (as many elements per wavefront as that).
+// With one or two elements (rules of many points, whose gradients fill LDS)
+// most lanes would have no tile: single pairs as long as they take at most
+// twice the rounds of the lanes.  Float32 blocks leave the lanes directly, and
+// a tile's are two blocks apart: single pairs there as well while the sums are
+// short.  Element kernel of linear elasticity, upper blocks, 2 x 2 / single
+// (us): 36^3 x 6 tetra, 5 points, float64, 353 / 137, 400^2 quads, 9 points,
+// 137 / 61 (59 before there were tiles); whole blocks with their reduction,
+// 12^3 x 6 tetra20, 4 points, float32, 138 / 116 (119), 24 points 253 / 270.
+constexpr int tile_side(int B, int L, int MQ, bool blocks_f32) {
+  const int nt = (B + 1) / 2, tiles = nt * (nt + 1) / 2, pairs = B * (B + 1) / 2;
+  const int r1 = (pairs + L - 1) / L, r2 = (tiles + L - 1) / L;
+  return r1 <= (L >= 32 ? 2 : 1) * r2 || (blocks_f32 && L >= 32 && MQ <= 16) ? 1 : 2;
+}
+
 // MQ: largest number of quadrature points the LDS arrays hold.  upper: only
 // the blocks i <= j (symmetric forms, TM_FLAG_UPPER); block (j, i) is always
 // stored as the exact transpose of block (i, j).  EPW elements per wavefront
 // on L = 64 / EPW lanes each, WPB wavefronts per workgroup; an element's
 // stages stay within its wavefront and need no workgroup barrier.
 //
-// Linear elasticity: a lane owns a 2 x 2 tile of node pairs and accumulates,
-// per pair, S[a][c] = sum_q jxw_q g_i[a] g_j[c]; the block is
+// Linear elasticity: a lane owns a tile of node pairs, 2 x 2 or a single one
+// (tile_side), and accumulates, per pair, S[a][c] = sum_q jxw_q g_i[a] g_j[c]; the block is
 //   lam S[a][c] + mu S[c][a] + mu delta_ac tr S,
 // 12 float64 operations per pair and point instead of 42 when the block is
 // formed at every point, and four gradients read from LDS for four pairs
@@ -59,7 +77,8 @@ __device__ __forceinline__ int64_t xcd_chunks(int64_t b, int64_t nb) {
 // and its gradients (1.5 KB) limit the wavefronts in flight.
 //
 // Scalar forms use the same tiles (upper ones only, a value stands for (i, j)
-// and (j, i)) and write the element's matrix from LDS: Laplace and diffusion
+// and (j, i)) and write the element's matrix from LDS, or single pairs of one
+// round from the lanes (mass on tetra10, 24 points, 57 -> 49 us): Laplace and diffusion
 // on hexahedra 40^3 float64 66 -> 46 us, tetra10 20^3 x 6 float32 44 -> 29 us.
 template <typename T, int D, int B, int H, int FORM, int MQ, int EPW, int WPB>
 __global__ void __launch_bounds__(kWave * WPB)
@@ -70,27 +89,42 @@ __global__ void __launch_bounds__(kWave * WPB)
   constexpr int L = kWave / EPW;   // lanes per element
   constexpr int kEpb = WPB * EPW;  // elements per workgroup
   constexpr bool kBlock = FORM == TM_FORM_LINEAR_ELASTICITY;
-  constexpr int NT = (B + 1) / 2;  // tiles per side
+  constexpr int TS = tile_side(B, L, MQ, kBlock && sizeof(T) == 4);  // nodes per side of a tile
+  constexpr int NT = (B + TS - 1) / TS;                               // tiles per side
+  constexpr int NP = TS * TS;                                         // pairs per tile
   __shared__ double s_tab[MQ * (1 + B + D * B)];
   __shared__ uint16_t s_tile[NT * NT];
-  __shared__ uint16_t s_pair[kBlock ? 1 : B * B];
-  // odd strides between elements: with even ones (192 doubles for hexahedra)
-  // the elements of a wavefront met in the same banks, half of all LDS cycles
-  __shared__ double s_jxw[kEpb][MQ | 1];
-  __shared__ double s_kq[kBlock ? 1 : kEpb][MQ | 1];
-  constexpr int kG = kBlock || MQ * D > B ? MQ * B * D : B * B;  // gradients, then a scalar form's matrix
-  __shared__ double s_g[kEpb][kG | 1];
+  // odd strides between many elements: with even ones (192 doubles for
+  // hexahedra) the elements of a wavefront met in the same banks, half of all
+  // LDS cycles.  With one or two elements even ones, which keep the reads of
+  // two gradient components 16-byte aligned (quads 400^2, 9 points, 70 -> 51 us).
+  constexpr int kOdd = EPW > 2 ? 1 : 0;
+  __shared__ double s_jxw[kEpb][MQ | kOdd];
+  __shared__ double s_kq[kBlock ? 1 : kEpb][MQ | kOdd];
+  // a scalar form of one round of single pairs stores its values from the lanes
+  constexpr bool kDirect = !kBlock && TS == 1 && NT * (NT + 1) / 2 <= L;
+  // gradients (none for the mass form), then a scalar form's matrix
+  constexpr int kGrad = FORM == TM_FORM_MASS ? 1 : MQ * B * D, kMat = kBlock || kDirect ? 1 : B * B;
+  __shared__ double s_g[kEpb][(kGrad > kMat ? kGrad : kMat) | kOdd];
+  __shared__ uint16_t s_pair[kBlock || kDirect ? 1 : B * B];
   __shared__ int s_v[FORM == TM_FORM_DIFFUSION_NODE ? kEpb : 1][B];
-  // with a point to at least half of an element's lanes, a point's lane goes
-  // from the coordinates to its gradients in registers; else the sums and the
-  // gradients are spread over the lanes, through inv
-  constexpr bool kFused = 2 * MQ >= L;
+  // with many elements per wavefront and points for more than half of an
+  // element's lanes, a point's lane goes from the coordinates to its gradients
+  // in registers; else the sums and the gradients are spread over the lanes,
+  // through inv (Laplace, us, in registers / spread: hexahedra 40^3, 27 points
+  // on 64 lanes, 237 / 198; tetra10 18^3 x 6 with the reduction, 5 points on 16
+  // lanes, 46.9 / 44.3)
+  constexpr bool kFused = 2 * MQ > L && EPW > 2;
   constexpr int kInv = kFused ? 0 : MQ * D * D;
   // what the blocks no longer need: each wavefront stages their stores there
   struct Early {
-    double x[(B * D + kInv) % 2 ? B * D : B * D + 1], inv[kFused ? 1 : MQ][kFused ? 1 : D * D];
+    double x[(B * D + kInv) % 2 == kOdd ? B * D : B * D + 1], inv[kFused ? 1 : MQ][kFused ? 1 : D * D];
   };
-  constexpr int kEarly = EPW * (int)sizeof(Early), kBlocks = kBlock ? tmh::stage_bytes<T, H * H>() : 0;
+  // Float64 blocks are stored through LDS, except a few per wavefront (36^3 x 6
+  // tetra, 5 points, two elements, 137 -> 110 us) and the 32-byte ones of four
+  // elements or less (quads of 9 nodes, whole blocks, two elements, 71 -> 64)
+  constexpr bool kStage = sizeof(T) == 8 && !(TS == 1 && B * (B + 1) <= L) && !(D == 2 && EPW <= 4);
+  constexpr int kEarly = EPW * (int)sizeof(Early), kBlocks = kBlock ? tmh::stage_bytes<T, H * H, kStage>() : 0;
   __shared__ __align__(16) char s_mem[WPB][kEarly > kBlocks ? kEarly : kBlocks];
 
   const int lane = threadIdx.x % kWave % L;          // lane within the element's group
@@ -115,7 +149,7 @@ __global__ void __launch_bounds__(kWave * WPB)
   // scalar forms compute the upper tiles only and store each value twice
   const int n_tiles = tmh::fill_pairs<NT>(s_tile, !kBlock || upper != 0);
   const int n_pairs = upper ? B * (B + 1) / 2 : B * B;
-  if constexpr (!kBlock) tmh::fill_pairs<B>(s_pair, upper != 0);
+  if constexpr (!kBlock && !kDirect) tmh::fill_pairs<B>(s_pair, upper != 0);
   const double* w = s_tab;
   const double* phi = s_tab + Q;
   const double* dphi = s_tab + Q + Q * B;
@@ -140,16 +174,16 @@ __global__ void __launch_bounds__(kWave * WPB)
     const int p = upper ? i * B - i * (i - 1) / 2 + j - i : i * B + j;
     return slot_dest ? slot_dest[e * n_pairs + p] : (int32_t)(e * n_pairs + p);
   };
-  auto tile_slots = [&](int t, int32_t (&d)[4], bool (&has)[4]) {
+  auto tile_slots = [&](int t, int32_t (&d)[NP], bool (&has)[NP]) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int i = 2 * (s_tile[t] >> 8) + k / 2, j = 2 * (s_tile[t] & 255) + k % 2;
+    for (int k = 0; k < NP; ++k) {
+      const int i = TS * (s_tile[t] >> 8) + k / TS, j = TS * (s_tile[t] & 255) + k % TS;
       has[k] = i < B && j < B && (!upper || i <= j);
       d[k] = has[k] ? pair_slot(i, j) : 0;
     }
   };
-  int32_t dst[4] = {0, 0, 0, 0};
-  bool has[4] = {false, false, false, false};
+  int32_t dst[NP] = {};
+  bool has[NP] = {};
   if constexpr (kBlock)
     if (active && lane < n_tiles) tile_slots(lane, dst, has);
   tmh::wave_sync();
@@ -191,6 +225,7 @@ __global__ void __launch_bounds__(kWave * WPB)
     }
   };
   auto gradient = [&](int q, int b, const double (&inv)[D][D]) {
+    if constexpr (FORM == TM_FORM_MASS) return;
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       double s = 0.0;
@@ -259,53 +294,61 @@ __global__ void __launch_bounds__(kWave * WPB)
       int I = mine ? s_tile[t] >> 8 : 0, J = mine ? s_tile[t] & 255 : 0;
       const bool low = I > J;
       if (t0 > 0) {
-        if (mine) tile_slots(t, dst, has);
-        else has[0] = has[1] = has[2] = has[3] = false;
+        if (mine) {
+          tile_slots(t, dst, has);
+        } else {
+#pragma unroll
+          for (int k = 0; k < NP; ++k) has[k] = false;
+        }
       }
       if (low) {
         const int u = I;
         I = J;
         J = u;
       }
-      const int i1 = 2 * I + 1 < B ? 2 * I + 1 : 2 * I, j1 = 2 * J + 1 < B ? 2 * J + 1 : 2 * J;
-      double S[4][HH];
+      // the tile's nodes, those past the last one standing in as the last
+      int ti[TS], tj[TS];
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
+      for (int k = 0; k < TS; ++k) {
+        ti[k] = TS * I + k < B ? TS * I + k : B - 1;
+        tj[k] = TS * J + k < B ? TS * J + k : B - 1;
+      }
+      double S[NP][HH];
+#pragma unroll
+      for (int k = 0; k < NP; ++k)
 #pragma unroll
         for (int n = 0; n < HH; ++n) S[k][n] = 0.0;
       for (int q = 0; q < Q; ++q) {
         const double* g = &s_g[wv][q * B * D];
         const double wq = s_jxw[wv][q];
-        double gi[2][D], gj[2][D];
+        double gi[TS][D], gj[TS][D];
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-          gi[0][d] = g[2 * I * D + d] * wq;
-          gi[1][d] = g[i1 * D + d] * wq;
-          gj[0][d] = g[2 * J * D + d];
-          gj[1][d] = g[j1 * D + d];
-        }
+        for (int k = 0; k < TS; ++k)
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+          for (int d = 0; d < D; ++d) {
+            gi[k][d] = g[ti[k] * D + d] * wq;
+            gj[k][d] = g[tj[k] * D + d];
+          }
+#pragma unroll
+        for (int k = 0; k < NP; ++k)
 #pragma unroll
           for (int a = 0; a < D; ++a)
 #pragma unroll
-            for (int c = 0; c < D; ++c) S[k][a * D + c] += gi[k / 2][a] * gj[k % 2][c];
+            for (int c = 0; c < D; ++c) S[k][a * D + c] += gi[k / TS][a] * gj[k % TS][c];
       }
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        // pair k of the tile as stored, (2I + k/2, 2J + k%2) before the swap:
-        // sums of pair (lo, hi), the diagonal tile's (1, 0) from its (0, 1)
-        const int kk = low ? (k % 2) * 2 + k / 2 : k;
+      for (int k = 0; k < NP; ++k) {
+        // pair k of the tile as stored, (TS I + k/TS, TS J + k%TS) before the
+        // swap: sums of pair (lo, hi), the diagonal tile's (1, 0) from its (0, 1)
+        constexpr int kTurn = TS == 2 ? 2 : -1;
+        const int mirror = (k % TS) * TS + k / TS;
+        const bool turned = k == kTurn && I == J;
         double s[HH];
 #pragma unroll
-        for (int n = 0; n < HH; ++n) {
-          const double a = S[k][n], b = S[(k % 2) * 2 + k / 2][n];
-          s[n] = kk == k ? a : b;
-          if (k == 2 && I == J) s[n] = S[1][n];
-        }
-        const bool flip = low || (k == 2 && I == J);
+        for (int n = 0; n < HH; ++n) s[n] = low || turned ? S[mirror][n] : S[k][n];
+        const bool flip = low || turned;
         // pair (i, i): the sums above the diagonal stand for those below
-        const bool self = I == J && k % 2 == k / 2;
+        const bool self = I == J && k % TS == k / TS;
 #pragma unroll
         for (int a = 0; a < D; ++a)
 #pragma unroll
@@ -323,7 +366,7 @@ __global__ void __launch_bounds__(kWave * WPB)
             blk[a * D + c] = v;
           }
         const bool neg = slot_dest && dst[k] < 0;   // contribution order: read as (j, i)
-        tmh::store_blocks<T, HH>(mem, blk, has[k] ? dst[k] & INT32_MAX : -1, flip != neg, slot);
+        tmh::store_blocks<T, HH, kStage>(mem, blk, has[k] ? dst[k] & INT32_MAX : -1, flip != neg, slot);
       }
     }
     return;
@@ -332,43 +375,69 @@ __global__ void __launch_bounds__(kWave * WPB)
   // the values of the lane's tiles, then the element's B x B matrix in the
   // place of its gradients, then contiguous stores
   constexpr int kRounds = (NT * (NT + 1) / 2 + L - 1) / L;
-  double S[kRounds][4];
+  double S[kRounds][NP];
 #pragma unroll
   for (int r = 0; r < kRounds; ++r) {
     const int t = lane + r * L;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) S[r][k] = 0.0;
+    for (int k = 0; k < NP; ++k) S[r][k] = 0.0;
     if (active && t < n_tiles) {
-      const int i0 = 2 * (s_tile[t] >> 8), j0 = 2 * (s_tile[t] & 255);
-      const int i1 = i0 + 1 < B ? i0 + 1 : i0, j1 = j0 + 1 < B ? j0 + 1 : j0;
+      int ti[TS], tj[TS];
+#pragma unroll
+      for (int k = 0; k < TS; ++k) {
+        const int i = TS * (s_tile[t] >> 8) + k, j = TS * (s_tile[t] & 255) + k;
+        ti[k] = i < B ? i : B - 1;
+        tj[k] = j < B ? j : B - 1;
+      }
       for (int q = 0; q < Q; ++q) {
         const double wq = s_jxw[wv][q];
         if constexpr (FORM == TM_FORM_MASS) {
           const double* ph = phi + q * B;
-          const double pi[2] = {ph[i0], ph[i1]}, pj[2] = {ph[j0], ph[j1]};
+          double pi[TS], pj[TS];
 #pragma unroll
-          for (int k = 0; k < 4; ++k) S[r][k] += (pi[k / 2] * pj[k % 2]) * wq;
+          for (int k = 0; k < TS; ++k) {
+            pi[k] = ph[ti[k]];
+            pj[k] = ph[tj[k]];
+          }
+#pragma unroll
+          for (int k = 0; k < NP; ++k) S[r][k] += (pi[k / TS] * pj[k % TS]) * wq;
         } else {
           const double* g = &s_g[wv][q * B * D];
           const double kq = s_kq[wv][q];
-          double gi[2][D], gj[2][D];
+          double gi[TS][D], gj[TS][D];
 #pragma unroll
-          for (int d = 0; d < D; ++d) {
-            gi[0][d] = g[i0 * D + d];
-            gi[1][d] = g[i1 * D + d];
-            gj[0][d] = g[j0 * D + d];
-            gj[1][d] = g[j1 * D + d];
-          }
+          for (int k = 0; k < TS; ++k)
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
+            for (int d = 0; d < D; ++d) {
+              gi[k][d] = g[ti[k] * D + d];
+              gj[k][d] = g[tj[k] * D + d];
+            }
+#pragma unroll
+          for (int k = 0; k < NP; ++k) {
             double dot = 0.0;
 #pragma unroll
-            for (int d = 0; d < D; ++d) dot += gi[k / 2][d] * gj[k % 2][d];
+            for (int d = 0; d < D; ++d) dot += gi[k / TS][d] * gj[k % TS][d];
             S[r][k] += (kq * dot) * wq;
           }
         }
       }
     }
+  }
+  T* out = slot + e * (int64_t)n_pairs;
+  if constexpr (kDirect) {
+    if (active && lane < n_tiles) {
+      const int i = s_tile[lane] >> 8, j = s_tile[lane] & 255;
+      const T v = (T)S[0][0];
+      if (!upper) {
+        out[i * B + j] = v;
+        out[j * B + i] = v;
+      } else if (slot_dest) {
+        slot[slot_dest[e * n_pairs + lane] & INT32_MAX] = v;
+      } else {
+        out[lane] = v;
+      }
+    }
+    return;
   }
   tmh::wave_sync();
   double* const mat = s_g[wv];
@@ -376,10 +445,10 @@ __global__ void __launch_bounds__(kWave * WPB)
   for (int r = 0; r < kRounds; ++r) {
     const int t = lane + r * L;
     if (active && t < n_tiles) {
-      const int i0 = 2 * (s_tile[t] >> 8), j0 = 2 * (s_tile[t] & 255);
+      const int i0 = TS * (s_tile[t] >> 8), j0 = TS * (s_tile[t] & 255);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int i = i0 + k / 2, j = j0 + k % 2;
+      for (int k = 0; k < NP; ++k) {
+        const int i = i0 + k / TS, j = j0 + k % TS;
         if (i < B && j < B) {
           mat[i * B + j] = S[r][k];
           mat[j * B + i] = S[r][k];
@@ -389,7 +458,6 @@ __global__ void __launch_bounds__(kWave * WPB)
   }
   tmh::wave_sync();
   if (!active) return;
-  T* out = slot + e * (int64_t)n_pairs;
   for (int p = lane; p < n_pairs; p += L) {
     const T v = (T)mat[upper ? (s_pair[p] >> 8) * B + (s_pair[p] & 255) : p];
     if (slot_dest)
@@ -893,12 +961,17 @@ int launch_wave(const tm_mesh_view* m, const tm_form_desc* f, void* slot_ws, hip
   constexpr int NT = (B + 1) / 2, kTiles = NT * (NT + 1) / 2;
   constexpr int kMost = kTiles >= kWave ? 1 : kWave / kTiles < 16 ? kWave / kTiles : 16;
   constexpr int kMany = kMost * kElemBytes <= 20480 ? kMost : kTwo;
-  const int epw = f->epw == 0 ? kMany : f->epw;
+  const int upper = (f->flags & TM_FLAG_UPPER) != 0;
+  // Whole blocks of the cells of 8 to 10 nodes: consecutive lanes on single
+  // pairs write consecutive blocks (element kernel and reduction, kMany / two:
+  // 18^3 x 6 tetra10 float32 109 / 90 us, hexahedra 40^3 119 / 97, float64
+  // 178 / 174 and 225 / 214).  Smaller cells lose by it (tetra 128 / 152).
+  constexpr int kWhole = B >= 8 && kMany > kTwo ? kTwo : kMany;
+  const int epw = f->epw != 0 ? f->epw : f->form == TM_FORM_LINEAR_ELASTICITY && !upper ? kWhole : kMany;
   if (epw != 1 && epw != kTwo && epw != kMany)
     return tmh::fail(TM_ERR_ARG, "elements per wavefront not admitted for this cell / rule");
   *hh_out = 1;
   double lam = 0.0, mu = 0.0;
-  const int upper = (f->flags & TM_FLAG_UPPER) != 0;
 #define TM_WAVE_E(H, FORM, EPW)                                                                                    \
   do {                                                                                                            \
     constexpr int kWpb = EPW * kWavesPerBlock * kElemBytes <= 40960 || EPW <= 2 ? kWavesPerBlock : 2;              \
