@@ -485,7 +485,7 @@ typedef float tm_floatx16 __attribute__((ext_vector_type(16)));
 // (e, i) (B blocks of D x D values) goes to e*B + i, or with inc_inv to its
 // position inc_inv[e*B + i] in the node-sorted incidence list.  In the VALU
 // tangent a lane forms a whole D x D block; float64 blocks are stored through
-// LDS, float32 ones from the lane (tmh::store_blocks).  The MFMA tile spreads a
+// LDS (kViaLds), float32 ones from the lane (tmh::store_blocks).  The MFMA tile spreads a
 // row over lanes, so that variant is staged in LDS and written as whole slot
 // rows with vector stores.
 // upper (TM_FLAG_UPPER): only the pairs i <= j.
@@ -518,7 +518,13 @@ __global__ void __launch_bounds__(kWave * (BIG ? 1 : kWavesPerBlock), TAN && !MF
   struct Early {
     double x[B * D], u[B * D], inv[MQ][D * D], P[MQ][D * D], Fi[MQ][D * D];
   };
-  constexpr int kEarly = EPW * (int)sizeof(Early), kBlocks = TAN && !MFMA ? tmh::stage_bytes<T, D * D>() : 0;
+  // Float64 blocks are stored through LDS, except few per wavefront and the
+  // large cells', whose lone wavefront waits for each of its rounds (assembly
+  // of residual and tangent, us, through LDS / from the lanes: 36^3 x 6 tetra,
+  // 4 points, 299 / 273; 12^3 x 6 tetra20, 24 points, 417 / 386; 18^3
+  // hexahedra of 27 nodes, 27 points, 487 / 449)
+  constexpr bool kViaLds = sizeof(T) == 8 && !BIG && B * (B + 1) > L;
+  constexpr int kEarly = EPW * (int)sizeof(Early), kBlocks = TAN && !MFMA ? tmh::stage_bytes<T, D * D, kViaLds>() : 0;
   __shared__ __align__(16) char s_mem[kWpb][kEarly > kBlocks ? kEarly : kBlocks];
   __shared__ double s_jxw[kEpb][kMaxQ];
   __shared__ double s_g[kEpb][kMaxQ * B * D];
@@ -773,7 +779,7 @@ __global__ void __launch_bounds__(kWave * (BIG ? 1 : kWavesPerBlock), TAN && !MF
     }
   } else if (ts) {
     // one lane per node pair (i, j): the whole D x D block from one read of
-    // g_i, g_j, h_i, h_j per quadrature point, stored through LDS
+    // g_i, g_j, h_i, h_j per quadrature point
     constexpr int DD = D * D;
     int32_t d_next = dst;
 #pragma unroll 1
@@ -831,7 +837,7 @@ __global__ void __launch_bounds__(kWave * (BIG ? 1 : kWavesPerBlock), TAN && !MF
             }
         }
       }
-      tmh::store_blocks<T, DD>(mem, acc, at, false, ts);
+      tmh::store_blocks<T, DD, kViaLds>(mem, acc, at, false, ts);
     }
   }
   if constexpr (kStage) {

@@ -2,7 +2,7 @@
 2 x 2 node pairs and single pairs, points in registers and spread over the
 lanes, stores through LDS and from the lanes.  Each against the oracle (the CPU
 path for the rule that it does not hold), and the same bits for every admitted
-number of elements per wavefront."""
+number of elements per wavefront.  Likewise the Neo-Hookean tangent's stores."""
 import pytest
 import torch
 
@@ -60,3 +60,28 @@ def test_rules(cell, q, form):
                 assert (got[None].cpu().double().reshape(want.shape) - want).abs().max() <= tol * want.abs().max()
                 for e, v in got.items():
                     assert torch.equal(v, got[None]), (dtype, sym, e)
+
+
+# cells with few blocks per wavefront, and those of one wavefront per workgroup
+@pytest.mark.parametrize("cell,q", [("triangle", 2), ("quad", 2), ("tetra", 2), ("tetra", 7), ("tetra20", 2), ("hexahedron27", 2)])
+def test_neo_hookean_blocks_from_the_lanes(cell, q):
+    m = {"triangle": lambda: unit_square_tri(3, 0.1, 1), "quad": lambda: unit_square_quad(3, 0.1, 1),
+         "tetra": lambda: unit_cube_tet(2, 0.1, 1), "tetra20": lambda: unit_cube_tet(1, 0.1, 1, order=3),
+         "hexahedron27": lambda: unit_cube_hex(1, 0.1, 1, order=2)}[cell]()
+    P, c, D = m.points, m.elements(), m.points.shape[1]
+    u = 0.03 * torch.stack([torch.sin(P[:, 1]), P[:, 0] * P[:, -1], 0.5 * P[:, 0] ** 2][:D], 1)
+    _, loc = fem.neohookean_element_tangent(P, c, cell, q, u, 1.0, 0.3)
+    want = torch.zeros(m.n_points, m.n_points, D, D, dtype=torch.float64)
+    want.index_put_((c[:, :, None].expand(-1, -1, c.shape[1]), c[:, None, :].expand(-1, c.shape[1], -1)), loc, accumulate=True)
+    want = want.permute(0, 2, 1, 3).reshape(D * m.n_points, -1)
+    A = tm.NeoHookeanModel.from_mesh(m.to(DEV), quadrature_order=q, E=1.0, nu=0.3)
+    for sym in (True, False):
+        A.symmetric_slots, first = sym, None
+        for epw in (None, 1, 2):
+            A.epw = epw
+            if epw == 2 and (cell in ("tetra20", "hexahedron27") or q == 7):
+                continue   # a wavefront takes one of these
+            _, K = A.residual_and_tangent(u.to(DEV))
+            assert (K.to_dense().cpu() - want).abs().max() <= 1e-12 * want.abs().max()
+            first = K.values if first is None else first
+            assert torch.equal(K.values, first)
