@@ -99,8 +99,9 @@ typedef struct tm_form_desc {
   double poisson;            /* LINEAR_ELASTICITY: nu */
   int32_t flags;             /* TM_FLAG_* */
   int32_t epw;               /* elements per wavefront of the wave kernels, 0 = the kernel's own choice:
-                                element matrices 1 or 2, Neo-Hookean 1, 2 or 4 (VALU tangent), J2 1, 4, 8
-                                or 16 (cells of <= 4 nodes with rules of <= 4 points); a count the cell,
+                                element matrices 1, 2 or that choice (4, 6, 10 or 16, by the cell's nodes,
+                                for rules of few points), Neo-Hookean 1, 2 or 4 (VALU tangent), J2 1, 4,
+                                8 or 16 (cells of <= 4 nodes with rules of <= 4 points); a count the cell,
                                 rule or LDS budget does not admit is TM_ERR_ARG.  Results do not depend
                                 on it (one lane group per element, the same arithmetic). */
 } tm_form_desc;

@@ -4,8 +4,8 @@
 ``reps`` more runs with device events, and keeps the fastest name per key;
 later calls (and later processes, through the JSON cache) reuse it without
 timing.  Keys name the device, the operation, the topology (the pattern's
-layout hash), the dtype and the form, so a choice is remade when any of
-them changes.
+layout hash), the dtype, the form and the revision of the kernels, so a choice
+is remade when any of them changes.
 
 The cache file is ``$TENSORMESH_AMD_TUNE_CACHE`` if set, else
 ``~/.cache/tensormesh_amd/tune.json``; if it cannot be written the tuner keeps
@@ -22,9 +22,10 @@ computation):
 * ``NeoHookeanModel.nh_path = "auto"``: slot-buffer segment reduction or
   incidence-ordered block rows; same element values, same order.
 * ``epw = "auto"`` on the element-matrix, Neo-Hookean and J2 assemblers:
-  elements per wavefront of the wave kernels (1/2, 1/2/4, 1/4/8; counts a
-  kernel does not admit for the case are skipped).  Each element keeps its
-  own lane group and arithmetic, so the results are bit-identical.
+  elements per wavefront of the wave kernels: the kernel's own choice for the
+  case (0, the first candidate) or 1/2, 1/2/4, 1/4/8/16; counts a kernel does
+  not admit are skipped.  Each element keeps its own lane group and
+  arithmetic, so the results are bit-identical.
 * ``BatchedPCG.solve(chunk=None)``: iterations per graph replay between
   convergence polls, from the previous solve's iteration count on the same
   system (systems stop on the device, so the chunk changes only the number of
@@ -42,6 +43,10 @@ from typing import Callable, Dict, Optional
 import torch
 
 _LOCK = threading.Lock()
+
+#: Counted up when a tuned kernel changes: choices timed on another revision,
+#: in this cache file or an older one, are timed again.
+KERNELS = 2
 
 
 def _cache_path() -> Path:
@@ -97,6 +102,7 @@ class Tuner:
                device: Optional[torch.device] = None) -> str:
         """Name of the fastest candidate for ``key`` (timed once, then cached)."""
         names = list(candidates)
+        key = f"{key}|k{KERNELS}"
         if not self.enabled or len(names) == 1:
             return names[0]
         hit = self.get(key)
