@@ -963,7 +963,10 @@ int launch_wave(const tm_mesh_view* m, const tm_form_desc* f, void* slot_ws, hip
   // else two where they fit 40 KB, else one.  form->epw: 1, 2 where two
   // elements' arrays fit, or the default (0)
   constexpr int kElemBytes = 8 * (B * D + MQ * (D * D + 2) + B * (MQ * D > B ? MQ * D : B)) + 4 * B;
-  constexpr int kTwo = (2 * kWavesPerBlock * kElemBytes <= 40960 && MQ <= kWave / 2 && B <= kWave / 2) ? 2 : 1;
+  // without a scalar form's matrix, which only the 27 nodes of a one-point rule
+  // outgrow the gradients by (59 KB of LDS for a workgroup of two elements)
+  constexpr int kGradBytes = 8 * (B * D + MQ * (D * D + 2 + B * D)) + 4 * B;
+  constexpr int kTwo = (2 * kWavesPerBlock * kGradBytes <= 40960 && MQ <= kWave / 2 && B <= kWave / 2) ? 2 : 1;
   constexpr int NT = (B + 1) / 2, kTiles = NT * (NT + 1) / 2;
   constexpr int kMost = kTiles >= kWave ? 1 : kWave / kTiles < 16 ? kWave / kTiles : 16;
   constexpr int kMany = kMost * kElemBytes <= 20480 ? kMost : kTwo;

@@ -7,7 +7,7 @@ import torch
 
 import tensormesh_amd as tm
 from tensormesh_amd import tune
-from tensormesh_amd.mesh import unit_cube_hex, unit_cube_tet
+from tensormesh_amd.mesh import unit_cube_hex, unit_cube_tet, unit_square_quad, unit_square_tri
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -41,3 +41,18 @@ def test_auto_times_the_default(dtype, tmp_path, monkeypatch):
         for e in timed:
             A.epw = int(e)
             assert torch.equal(run(A), want), (kernel, e)
+
+
+@pytest.mark.parametrize("cell", ["triangle6", "triangle10", "tetra10", "tetra20", "quad", "quad9", "hexahedron", "hexahedron27"])
+def test_two_elements_are_admitted_for_short_rules(cell):
+    """One-point rules leave room for two elements of every cell."""
+    print(f"case two elements {cell}", flush=True)
+    order = 2 if cell[-1] in "69" or cell in ("tetra10", "hexahedron27") else 3 if cell[-2:] in ("10", "20") else 1
+    make = {"tri": unit_square_tri, "tet": unit_cube_tet, "qua": unit_square_quad, "hex": unit_cube_hex}[cell[:3]]
+    m = make(2, 0.1, 1, order=order).to(DEV)
+    assert list(m.cells) == [cell]
+    for A in (tm.MassElementAssembler.from_mesh(m, quadrature_order=1),
+              tm.LinearElasticityElementAssembler.from_mesh(m, quadrature_order=1, E=1.0, nu=0.3)):
+        want = A().values
+        for A.epw in (1, 2):
+            assert torch.equal(A().values, want)
