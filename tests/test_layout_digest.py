@@ -71,4 +71,41 @@ def test_a_moved_condenser_lets_go_of_its_indices():
     assert here == [id(cond.inner_row), id(cond.inner_col)]
     cond.to("meta")
     assert all(i.device.type == "meta" for i in cond._inner_hash._index)
+    assert cond.layout_hash == _want(K) and not isinstance(vars(cond).get("_layout"), LazyDigest)
     assert Ki.layout_hash == _want(Ki)
+
+
+def test_condensing_the_same_indices_hashes_nothing(digests):
+    m, A, K = _block_matrix()
+    f = torch.ones(K.shape[0], dtype=torch.float64)
+    cond = tm.Condenser(m.boundary_mask.repeat_interleave(2))
+    assert cond.layout_hash is None
+    cond(K, f)
+    cond(A(), f)
+    cond(K.detach(), f)
+    assert A().has_same_layout(K) and not digests
+    same = SparseMatrix(K.values, K.row_indices.clone(), K.col_indices.clone(), K.shape)
+    cond(same, f)                                   # other tensors: compared by digest
+    assert cond.layout_hash == _want(K) and len(digests) == 2
+    other = SparseMatrix(K.values, K.row_indices, K.col_indices.flip(0), K.shape)
+    with pytest.raises(AssertionError, match="layout of the matrix is changed"):
+        cond(other, f)
+    _, _, K5 = _block_matrix(5)
+    assert not K5.has_same_layout(K) and not K.has_same_layout(K5) and K.has_same_layout(_want(K))
+    with pytest.raises(TypeError):
+        K.has_same_layout(None)
+
+
+def test_condenser_files(digests):
+    m, _, K = _block_matrix()
+    f = torch.ones(K.shape[0], dtype=torch.float64)
+    cond = tm.Condenser(m.boundary_mask.repeat_interleave(2))
+    cond(K, f)
+    state = cond.__getstate__() if hasattr(cond, "__getstate__") else cond.__dict__
+    old = dict(state, layout_hash=_want(K))         # as written before digests were computed on demand
+    del old["_layout"]
+    older = tm.Condenser.__new__(tm.Condenser)
+    older.__setstate__(old)
+    for c in (older, _saved(cond), copy.deepcopy(cond)):
+        assert c.layout_hash == _want(K)
+        c(K, f)
