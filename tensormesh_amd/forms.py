@@ -185,8 +185,9 @@ def _owner_key(obj, depth: int, seen: set):
         return ("seen", id(obj))
     seen.add(id(obj))
     out = []
-    # the private attributes are most of them: out before the sort
-    for k, v in sorted([kv for kv in obj.__dict__.items() if not kv[0].startswith("_") or kv[0] in _OWNED]):
+    # the private attributes are most of them: out before the sort (of a copy of
+    # the items: another thread's first call adds attributes meanwhile)
+    for k, v in sorted([kv for kv in list(obj.__dict__.items()) if not kv[0].startswith("_") or kv[0] in _OWNED]):
         if k in ("_parameters", "_buffers"):
             out.extend((f"{k}.{n}", _value_key(t, depth, seen)) for n, t in v.items() if t is not None)
         elif k == "_modules":
