@@ -44,7 +44,8 @@ __device__ __forceinline__ void wave_sync() {
 // cycles per 64 lanes of 16 bytes (Neo-Hookean tetra10: 1.75e8 of its cycles
 // against 1.20e8 staged, 60 M write requests to L2 against 23 M, kernel
 // 398 -> 360 us).  Float32 blocks are half that and leave the lanes directly:
-// staged, the same kernel went from 133 to 141 us at 24^3 x 6 elements.
+// staged, the same kernel went from 133 to 141 us at 24^3 x 6 elements.  STAGE
+// = false: callers whose lanes hold few blocks, or small ones, at a time.
 // stage: stage_bytes<T, N>() bytes of LDS of this wavefront.
 constexpr int kStageBlocks = 32;
 template <typename T, int N, bool STAGE = sizeof(T) == 8>

@@ -1,22 +1,24 @@
-// Stage G for quadratic simplices and block (vector) forms: one wavefront per
-// element.
+// Stage G for every cell but the scalar P1 forms: element matrices
+// (wave_element_kernel) and the Neo-Hookean residual and tangent
+// (hyper_wave_kernel), one or more elements per wavefront.
 //
 // Replaces the same reference chain as tm_p1.hip -- eval_shape_grad
 // (tensormesh/element/element.py:956-968), jxw (transformation.py:1265-1272),
 // the vmap'd forward and _integrate (element_assembler.py:190-209,416-438) --
-// for triangle6 / tetra10 and for LinearElasticityElementAssembler
-// (builtin.py:172-178), where the Jacobian varies per quadrature point and a
-// local matrix has up to 30 x 30 entries.
+// for triangle6 / tetra10 and larger cells and for
+// LinearElasticityElementAssembler (builtin.py:172-178), where the Jacobian
+// varies per quadrature point and a local matrix has up to 81 x 81 entries.
 //
-// Work split inside the wave:
+// Work split among an element's lanes:
 //   1. lanes load the element's B*D coordinates into LDS;
-//   2. lane q builds J_q[i][j] = sum_b x[b][j] dphi_q[i][b], its inverse and
-//      jxw_q = w_q |det J_q|;
-//   3. lanes over (q, b, d) form grad_q[b][d] = sum_i dphi_q[i][b] Jinv_q[d][i];
-//   4. lanes stride over the B*B*H*H local entries; entry (i, j, a, c) is
-//      sum_q jxw_q * f_q(i, j, a, c) and is written to the slot buffer at
-//      ((e*B + i)*B + j)*H*H + a*H + c, the flattening of the reference's
-//      [E, B, B, H, H] element tensor.
+//   2. J_q[i][j] = sum_b x[b][j] dphi_q[i][b], its inverse and
+//      jxw_q = w_q |det J_q|, by point q's lane or with the sums spread over
+//      the lanes;
+//   3. grad_q[b][d] = sum_i dphi_q[i][b] Jinv_q[d][i] into LDS;
+//   4. lanes take tiles of node pairs (i, j); a pair's H x H block, from sums
+//      over the points, is written to slot (e*B + i)*B + j -- the flattening of
+//      the reference's [E, B, B, H, H] element tensor -- or packed, or in
+//      contribution order (TM_FLAG_UPPER, slot_dest).
 // Linear elasticity uses Ba^T C Bb in closed form:
 //   (Ba^T C Bb)[a][c] = lam g_i[a] g_j[c] + mu g_i[c] g_j[a] + mu delta_ac g_i.g_j
 // which is the product of the Voigt matrices of functional/elasticity.py:132-284.
@@ -562,7 +564,7 @@ __global__ void __launch_bounds__(kWave * (BIG ? 1 : kWavesPerBlock), TAN && !MF
     }
   }
   tmh::wave_sync();
-  // the Jacobians J[i][j] = sum_b dphi_b[i] x_b[j] (into s_inv, which
+  // the Jacobians J[i][j] = sum_b dphi_b[i] x_b[j] (into el.inv, which
   // point q's lane then overwrites with the inverse)
   if (active)
     tmh::point_sums<D, B, L, MQ>(
@@ -626,7 +628,7 @@ __global__ void __launch_bounds__(kWave * (BIG ? 1 : kWavesPerBlock), TAN && !MF
   }
   tmh::wave_sync();
   // the deformation gradients F[a][d] = delta_ad + sum_b u_b[a] g_b[d] (into
-  // s_Fi, which the per-point stage below overwrites with F^-1)
+  // el.Fi, which the per-point stage below overwrites with F^-1)
   if (active)
     tmh::point_sums<D, B, L, MQ>(
         lane, Q, true, [&](int, int a, int b) { return el.u[b * D + a]; },
@@ -960,8 +962,8 @@ int launch_wave(const tm_mesh_view* m, const tm_form_desc* f, void* slot_ws, hip
   // By default as many elements per wavefront as have a lane for every tile
   // of the upper triangle (at most 16), where a wavefront's arrays fit 20 KB,
   // in workgroups of two wavefronts where four would take more than 40 KB;
-  // else two where they fit 40 KB, else one.  form->epw: 1, 2 where two
-  // elements' arrays fit, or the default (0)
+  // else two where their gradients fit 40 KB, else one.  form->epw: 1, two where
+  // that holds, or the default (0)
   constexpr int kElemBytes = 8 * (B * D + MQ * (D * D + 2) + B * (MQ * D > B ? MQ * D : B)) + 4 * B;
   // without a scalar form's matrix, which only the 27 nodes of a one-point rule
   // outgrow the gradients by (59 KB of LDS for a workgroup of two elements)

@@ -26,9 +26,12 @@
 // k publishes in buffer k mod 3 and resets buffer (k + 1) mod 3, last read in
 // step k - 2; a workgroup publishes its sums of step k only after its reset
 // has reached memory, and nobody reads buffer (k + 1) before it has
-// everybody's sums of step k.  Relaxed agent-scope accesses suffice (they go
-// past the caches of one XCD); a release store instead writes the whole L2
-// back, which took 21.6 us per step.  u of other workgroups' rows (the halo) is
+// everybody's sums of step k.  The accesses are relaxed at agent scope: on this
+// chip they go past the caches of one XCD, and a store counted off by
+// s_waitcnt vmcnt has reached the memory that all XCDs read.  That property,
+// not the language's memory model, orders the reset before the sums; a release
+// store would order it too, but writes the whole L2 back (10 of the 21.6 us
+// that a step then took).  u of other workgroups' rows (the halo) is
 // read once per workgroup into LDS: gathered from memory per matrix entry it
 // took 11.8 us.  Every workgroup adds its system's partial sums itself, in
 // workgroup order, so all of them take the same decisions without a broadcast
@@ -37,7 +40,9 @@
 // The workgroups of a launch that exchange through memory are co-resident by
 // a cooperative launch, and every wait is bounded: after kGiveUpTicks a
 // workgroup raises the abort word and leaves, as do all that see it or time
-// out themselves; the caller then solves with the two-launch kernels.
+// out themselves; the caller then solves with the two-launch kernels.  So does
+// a workgroup that cannot hold what it was given: too many halo columns, a row
+// of more entries than the instance's, a column of another system.
 #include <hip/hip_runtime.h>
 
 #include "tm_device.h"
