@@ -125,3 +125,30 @@ def test_no_memory_for_the_workspace(monkeypatch):
     for x, y in zip(b.solve(f), want):
         assert torch.equal(x, y)
     assert b._run is None
+
+
+@pytest.mark.parametrize("bad", [0, 2])   # the system whose last row is too long: in the first group, in the last
+def test_one_of_several_groups_ends_without_a_result(bad, monkeypatch):
+    """Groups launched after one that ended, and before it: all are solved again."""
+    print(f"case groups {bad}", flush=True)
+    systems = [_laplace(unit_square_tri(n, 0.2, n)) for n in (70, 60, 50)]
+    rows, cols, vals, offs = [], [], [], [0]
+    for k, (K, _) in enumerate(systems):
+        N = K.shape[0]
+        r, c, v = K.row_indices, K.col_indices, K.values
+        if k == bad:   # nine more entries, zeros, on the last row
+            r = torch.cat([r, torch.full((9,), N - 1, device=DEV)])
+            c = torch.cat([c, torch.arange(9, device=DEV)])
+            v = torch.cat([v, torch.zeros(9, dtype=torch.float64, device=DEV)])
+            order = torch.argsort(r * N + c)
+            r, c, v = r[order], c[order], v[order]
+        rows.append(r + offs[-1]); cols.append(c + offs[-1]); vals.append(v); offs.append(offs[-1] + N)
+    rp = torch.zeros(offs[-1] + 1, dtype=torch.int64, device=DEV)
+    rp[1:] = torch.cumsum(torch.bincount(torch.cat(rows), minlength=offs[-1]), 0)
+    a, b = (BatchedPCG(rp, torch.cat(cols), torch.cat(vals), offs, rtol=1e-10) for _ in range(2))
+    f = torch.cat([f for _, f in systems])
+    want = a.solve(f, chunk=32)
+    wgs = -(-np.diff(b._sys_blk) // 4)
+    b._run = b._make_plan(1, 8, int(wgs.max()), wgs)
+    assert b._run.n_launch == 3
+    _falls_back(b, f, want)
